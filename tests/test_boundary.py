@@ -1,6 +1,9 @@
 """CPU checks of the drop-in boundary: the C ABI library, op schemas and meta rules, the
 converter extension surface and the Dynamo backend on the CPU debug path."""
+import os
 import re
+import subprocess
+import sys
 from pathlib import Path
 
 import numpy as np
@@ -55,6 +58,32 @@ def test_library_rejects_bad_arguments_without_gpu():
     with pytest.raises(RuntimeError, match="drop-pad"):
         _lib.call("tai_moe_finalize_routing", 1, 15, 4, 8, 2, None, None, None, None, -1, 1, None, 1, 1, None)
     assert _lib.query("tai_grouped_matmul_workspace_size", 32768, 4096, 256) > 0
+
+
+def test_quant_matmul_plans_every_short_k_on_the_host():
+    """K below one 64-byte stage has no split plan: the host path must get past the planning to a launch, which
+    fails here for want of a device (in a process of its own: a division by zero there ends the process)."""
+    if torch.cuda.is_available():
+        pytest.skip("host buffers: only without a device")
+    code = """
+import torch
+from torchair_amd import _lib
+buf = torch.zeros(1 << 20, dtype=torch.int32)
+for m in (255, 256, 300, 5000):
+    for k in (16, 32, 48, 64, 80):
+        for layout in (_lib.LAYOUT_KN, _lib.LAYOUT_NK):
+            for out in (_lib.DT_INT32, _lib.DT_BF16, _lib.DT_INT8):
+                try:
+                    _lib.call("tai_quant_matmul", buf.data_ptr(), buf.data_ptr(), m, k, 512, layout, buf.data_ptr(), 1,
+                              None, 0, None, None, _lib.DT_NONE, out, buf.data_ptr(), buf.data_ptr(), 1 << 40, None)
+                except _lib.KernelError as e:
+                    assert "launch failed" in str(e), e
+                else:
+                    raise AssertionError("launched without a device")
+"""
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True,
+                       env={**os.environ, "PYTHONPATH": str(ROOT), "HIP_VISIBLE_DEVICES": "-1"})
+    assert r.returncode == 0, (r.returncode, r.stderr[-2000:])
 
 
 def test_ops_refuse_cpu_tensors_without_the_debug_path():

@@ -42,3 +42,24 @@ def test_no_workspace():
     _lib.call("tai_quant_matmul", x.data_ptr(), w.data_ptr(), m, k, n, _lib.LAYOUT_KN, None, 0, None, 0, None, None,
               _lib.DT_NONE, _lib.DT_INT32, out.data_ptr(), None, 0, torch.cuda.current_stream().cuda_stream)
     assert torch.equal(out.double(), x.double() @ w.double())
+
+
+@pytest.mark.parametrize("m", [256, 300])
+@pytest.mark.parametrize("k", [16, 32, 48])
+@pytest.mark.parametrize("nk", [False, True])
+def test_short_k(m, k, nk):
+    """K below one 64-byte stage, which no split plan takes: the 128-row tiles, with every output type."""
+    n = 512
+    g = torch.Generator(device=DEV).manual_seed(m + k)
+    x = torch.randint(-128, 128, (m, k), generator=g, device=DEV, dtype=torch.int8)
+    w = torch.randint(-128, 128, (k, n), generator=g, device=DEV, dtype=torch.int8)
+    wt = w.t().contiguous().t() if nk else w
+    want = x.double() @ w.double()
+    print("case", m, k, nk, flush=True)
+    acc = torch.ops.npu.npu_quant_matmul(x, wt, torch.ones(1, device=DEV), output_dtype=torch.int32)
+    assert torch.equal(acc.double(), want)
+    scale = torch.rand(n, generator=g, device=DEV) * 1e-3
+    y = torch.ops.npu.npu_quant_matmul(x, wt, scale, output_dtype=torch.bfloat16)
+    assert torch.equal(y, (acc.float() * scale).to(torch.bfloat16))
+    y8 = torch.ops.npu.npu_quant_matmul(x, wt, scale, output_dtype=torch.int8)
+    assert torch.equal(y8, (acc.float() * scale).round().clamp(-128, 127).to(torch.int8))

@@ -1239,7 +1239,7 @@ SplitPlan skinny_plan(int64_t m, int64_t k, int64_t n) {
     const double us = 0.45 * static_cast<double>(cdiv(nk, s)) + 3.0 + static_cast<double>(m) * n * s * 8 / 5e6;
     if (us < best) { best = us; want = s; }
   }
-  p.per = cdiv(nk, want);
+  p.per = imax64(1, cdiv(nk, want));
   p.split = cdiv(nk, p.per);
   return p;
 }
@@ -1808,12 +1808,14 @@ static int quant_matmul_impl(const int8_t* x1, const int8_t* x2, int64_t m, int6
     }
     return launch_status("tai_quant_matmul");
   }
-  // From 256 rows on, a caller without room for the partials gets the 256 x 256 tiles.
-  const bool split_room = m < 256 || skinny_plan(m, k, n).split == 1 ||
+  // A plan exists only for what skinny_ok takes (a K below one stage has none). From 256 rows on, a caller without
+  // room for the partials gets the 256 x 256 tiles.
+  const bool skinny = skinny_ok(m, k, n, x2_layout) && cfg_available<SkinnyCfg>();
+  const SplitPlan p = skinny ? skinny_plan(m, k, n) : SplitPlan{};
+  const bool split_room = m < 256 || p.split == 1 ||
                           (workspace != nullptr && ws_bytes >= quant_matmul_ws_base(m, k, n) &&
                            (reinterpret_cast<uintptr_t>(workspace) % 16) == 0);
-  if (skinny_ok(m, k, n, x2_layout) && split_room && cfg_available<SkinnyCfg>()) {
-    const SplitPlan p = skinny_plan(m, k, n);
+  if (skinny && split_room) {
     g.m_slots = p.m_slots;
     g.n_tiles = p.n_tiles;
     if (p.split == 1) {
