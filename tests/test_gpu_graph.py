@@ -4,7 +4,9 @@ group lists, cache slots) are checked against eager and the oracle on every repl
 work and synchronisations in between. This is the role of the reference's graph_task_update
 (python/torchair/_acl_concrete_graph/acl_graph.py:542-577): data-dependent sizes are read on the
 device, so a replay with new values needs no re-capture."""
+import gc
 import math
+import weakref
 
 import numpy as np
 import pytest
@@ -404,3 +406,44 @@ def test_compiled_int8_cache_and_sink_decode_replay_with_new_lengths():
             _churn()
         assert tai_graph.stats["captures"] == caps + 1
         assert tai_graph.stats["eager_fallbacks"] == falls
+
+
+def _cyclic_runner(x):
+    """A captured runner whose function refers back to what holds it."""
+    held = {}
+    held["runner"] = tai_graph.HipGraphRunner(lambda t: (held, torch.ops.npu.npu_dynamic_quant(t)[0])[1],
+                                              clone_input=False)
+    held["runner"](x)
+    return held
+
+
+def test_a_dropped_graph_outlives_the_capture_of_the_next():
+    """A runner whose function refers back to it is left to the cyclic collector; dropped just as another capture
+    begins, with the collector due at the next allocations, its graph is freed after that capture, and the new
+    graph replays as eager."""
+    x = torch.randn(64, 512, device=DEV).to(torch.bfloat16)
+    box, seen, threshold = [_cyclic_runner(x)], [], gc.get_threshold()
+    gone = weakref.ref(next(iter(box[0]["runner"].graphs.values())))
+
+    def step(t):
+        if torch.cuda.is_current_stream_capturing():
+            box.clear()
+            gc.set_threshold(1, 1, 1)
+            keep = [[i] for i in range(3000)]
+            seen.append(len(keep) == 3000 and gone() is not None)
+        return torch.ops.npu.npu_dynamic_quant(t)
+
+    runner = tai_graph.HipGraphRunner(step, clone_input=False)
+    try:
+        runner(x)
+    finally:
+        gc.set_threshold(*threshold)
+    assert seen == [True]
+    gc.collect()
+    assert gone() is None
+    for _ in range(3):
+        x.copy_(torch.randn(64, 512, device=DEV).to(torch.bfloat16))
+        _churn()
+        q, s = runner(x)
+        wq, ws = torch.ops.npu.npu_dynamic_quant(x)
+        assert torch.equal(q, wq) and torch.equal(s, ws)

@@ -9,6 +9,8 @@ tensors read by the kernels, so a replay with new values needs no re-capture.
 """
 from __future__ import annotations
 
+import contextlib
+import gc
 import logging
 import threading
 from typing import Any, Callable, Dict, List, Sequence, Tuple
@@ -36,6 +38,31 @@ def capture_resources():
     (None outside a capture). Ops keep what a captured graph reads at replay time (pinned buffers)
     there, so it lives exactly as long as that graph."""
     return getattr(_state, "resources", None)
+
+
+_collector_lock = threading.Lock()
+_collector = {"captures": 0, "was_on": False}
+
+
+@contextlib.contextmanager
+def _collector_off():
+    """Keeps Python's cyclic collector off while a graph is captured, and puts it back as it was when the last of
+    the captures under way ends. A dropped runner is often part of a cycle (its function refers to the program's
+    state, which holds the runner), so its graphs wait for the collector, which runs whenever enough containers have
+    been allocated: also inside the next capture. Destroying a graph synchronises the device; that is not allowed
+    while a stream captures (on any thread), and the error, raised in a destructor, ends the process."""
+    with _collector_lock:
+        if _collector["captures"] == 0:
+            _collector["was_on"] = gc.isenabled()
+            gc.disable()
+        _collector["captures"] += 1
+    try:
+        yield
+    finally:
+        with _collector_lock:
+            _collector["captures"] -= 1
+            if _collector["captures"] == 0 and _collector["was_on"]:
+                gc.enable()
 
 
 def _signature(args: Sequence[Any], pinned: Sequence[bool]) -> Tuple:
@@ -92,7 +119,7 @@ class _Captured:
                 _state.warmup = False
         torch.cuda.current_stream(dev).wait_stream(side)
         self.graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(self.graph):
+        with _collector_off(), torch.cuda.graph(self.graph):
             out = fn(*self.inputs)
         self.outputs = out
 
