@@ -266,3 +266,31 @@ def test_packed_rows_off_16_bytes_take_the_general_kernel(monkeypatch):
     assert sizes[-1] == 0
     _assert_same(call(wide[..., 1:].contiguous()), off, 4.5)
     assert sizes[-1] > 0
+
+
+@pytest.mark.parametrize("bs", [32, 96])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_packed_band_does_not_read_released_pages(bs, dt):
+    """A sliding window whose lower edge lies inside a 64-token tile but past that tile's first page: pages below the
+    band may have left the block table. They name a page of NaN and infinities here, whose values would send the
+    block to the plain fp32 path; the result equals, bit for bit, that with the pages still in the table."""
+    g = torch.Generator().manual_seed(370 + bs)
+    hq, hkv, d, pre = 8, 2, 128, 130
+    lq, lk = [1, 5, 70], [231, 1000, 560]  # lower edges at 100, 865 and 360
+    bt, n = _table(lk, bs, g)
+    k, v = _kv(n, bs, hkv, d, dt, g)
+    spare = (set(range(n)) - {int(p) for row, m in zip(bt, lk) for p in row[:-(-m // bs)]}).pop()
+    k[spare], v[spare] = math.nan, math.inf
+    q = torch.randn(sum(lq), hq, d, generator=g).to(dt).to(DEV)
+    gone = bt.clone()
+    for b, (nq, nk) in enumerate(zip(lq, lk)):
+        gone[b, :(nk - nq - pre) // bs] = spare
+    assert (gone != bt).any(1).all()
+    print("case", bs, dt, flush=True)
+    call = lambda t: FIA(q, k, v, actual_seq_lengths=torch.tensor(np.cumsum(lq), device=DEV),  # noqa: E731
+                         actual_seq_lengths_kv=torch.tensor(lk, device=DEV), block_table=t.to(DEV), num_heads=hq,
+                         num_key_value_heads=hkv, input_layout="TND", block_size=bs, scale=d ** -0.5, sparse_mode=4,
+                         pre_tokens=pre, next_tokens=0, softmax_lse_flag=True)
+    want, got = call(bt), call(gone)
+    assert np.isfinite(want[0].float().cpu().numpy()).all()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])

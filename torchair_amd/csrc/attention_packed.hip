@@ -257,21 +257,26 @@ __device__ __forceinline__ void packed_segment(const PackedArgs& p, char* smem, 
   const int bs = static_cast<int>(a.block_size);
   const int kstr = static_cast<int>(a.k1_strides[1]), vstr = static_cast<int>(a.v_strides[1]);
   const int lk = static_cast<int>(s.lk);
-  // tile u of the segment -> ring slot u % 4; rows past the sequence's end load its last row
+  const int lowest = rel(vis_lo(p, s, static_cast<uint32_t>(j) * kKCols / g));  // the block's lowest visible token
+  // tile u of the segment -> ring slot u % 4; rows past the sequence's end load its last row, rows below the band
+  // the lowest token that the block sees
   auto issue = [&](int u) __attribute__((always_inline)) {
     char* kst = smem + (u % kPStages) * 2 * T::kTile;
-    const int t0 = static_cast<int>(base) + u * kPKV;
+    const int t0 = static_cast<int>(base) + u * kPKV, first = max(0, lowest - u * kPKV);
     // a tile spans at most two pages (block_size >= 32, a multiple of 32): page ids through the scalar cache, whose
     // wait leaves the ring's loads alone
     int split = kPKV;  // rows from here on lie in the second page
-    int64_t k0, v0, k1 = 0, v1 = 0;
+    int64_t k0 = 0, v0 = 0, k1 = 0, v1 = 0;
     if (btrow) {
       const int pg = t0 / bs, slot0 = t0 - pg * bs;
-      const int64_t id0 = sload_i32(btrow + pg);
-      k0 = id0 * a.k1_strides[0] + static_cast<int64_t>(slot0) * kstr;
-      v0 = id0 * a.v_strides[0] + static_cast<int64_t>(slot0) * vstr;
-      if (slot0 + kPKV > bs && t0 + (bs - slot0) < lk) {
-        split = bs - slot0;
+      const bool two = slot0 + kPKV > bs && t0 + (bs - slot0) < lk;
+      if (two) split = bs - slot0;
+      if (first < split) {  // (a page wholly below the band may have left the table)
+        const int64_t id0 = sload_i32(btrow + pg);
+        k0 = id0 * a.k1_strides[0] + static_cast<int64_t>(slot0) * kstr;
+        v0 = id0 * a.v_strides[0] + static_cast<int64_t>(slot0) * vstr;
+      }
+      if (two) {
         const int64_t id1 = sload_i32(btrow + pg + 1);
         k1 = id1 * a.k1_strides[0] - static_cast<int64_t>(split) * kstr;
         v1 = id1 * a.v_strides[0] - static_cast<int64_t>(split) * vstr;
@@ -286,7 +291,7 @@ __device__ __forceinline__ void packed_segment(const PackedArgs& p, char* smem, 
       const int q = w * T::kLoadsPerWave + i;
       const int r = q * T::kRpi + lane / T::kCpr;
       const int ch = (lane % T::kCpr) ^ T::swz(r);
-      const int rr = min(r, last);
+      const int rr = min(max(r, first), last);
       const int64_t ko = (rr < split ? k0 : k1) + static_cast<int64_t>(rr * kstr + 8 * ch);
       const int64_t vo = (rr < split ? v0 : v1) + static_cast<int64_t>(rr * vstr + 8 * ch);
       __builtin_amdgcn_global_load_lds((gbl_void_t*)(kbase + ko), (lds_void_t*)(kst + q * 1024), 16, 0, 0);
