@@ -14,7 +14,7 @@ DEV = "cuda"
 
 
 @pytest.mark.parametrize("t", [1, 256, 257])
-@pytest.mark.parametrize("h,k", [(8, 1), (504, 8), (520, 9), (7168, 8), (520, 17)])
+@pytest.mark.parametrize("h,k", [(8, 1), (520, 2), (520, 3), (520, 4), (520, 5), (504, 8), (520, 9), (7168, 8), (520, 17)])
 def test_finalize_sizes(t, h, k):
     g = torch.Generator().manual_seed(t + h + k)
     ex = torch.randn(t * k + 1, h, generator=g).to(torch.bfloat16)
