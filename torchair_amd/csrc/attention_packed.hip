@@ -579,11 +579,14 @@ __global__ __launch_bounds__(256) void packed_merge_kernel(PackedArgs p) {
   const tai_fia_general_args& a = p.a;
   const int tid = threadIdx.x, lane = tid & 63;
   if (blockIdx.x >= 8 * kKWgs) {
+    // a lane looks at each of the 64 rows (one after another they took 5 us where all belonged to a sequence: 64
+    // single tokens over 500 keys, 16 / 8 heads of 64, 42.1 us then, 36.8 now)
     const int64_t rows = a.q_cum ? a.s_q : a.b * a.s_q, v0 = (static_cast<int64_t>(blockIdx.x) - 8 * kKWgs) * 64;
-    const int64_t end = a.q_cum ? a.q_cum[a.b - 1] : 0;
-    for (int64_t v = v0; v < imin64(v0 + 64, rows); ++v) {
+    const int64_t vl = v0 + lane, bl = a.q_cum ? 0 : vl / a.s_q;
+    const bool spare = vl < rows && (a.q_cum ? vl >= a.q_cum[a.b - 1] : a.seq_lens_q && vl - bl * a.s_q >= a.seq_lens_q[bl]);
+    for (uint64_t todo = __ballot(spare); todo; todo &= todo - 1) {
+      const int64_t v = v0 + __ffsll(static_cast<unsigned long long>(todo)) - 1;
       const int64_t b = a.q_cum ? 0 : v / a.s_q, i = v - b * a.s_q;
-      if (a.q_cum ? v < end : (!a.seq_lens_q || i < a.seq_lens_q[b])) continue;
       for (int e = 4 * tid; e < a.hq * D; e += 1024) {
         const int head = e / D;
         *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.out) + b * a.out_strides[0] + i * a.out_strides[1] +
