@@ -203,6 +203,13 @@ def test_mla_cfg5():
     _check_mla(lens, 128, 128, 122)
 
 
+@pytest.mark.parametrize("n,h", [(32, 16), (33, 16), (70, 64), (33, 65)])
+def test_mla_many_sequences(n, h):
+    """Around the batch and head counts where the charge for a sequence's start changes: many sequences that begin
+    inside a workgroup's range, empty ones and one-token ones among them."""
+    _check_mla([(37 * i) % 190 for i in range(n)], h, 64, 126 + n + h)
+
+
 def test_mla_rising_logits_take_the_rescaling_pass():
     # Every third page of sequence 0 has rope keys whose logits exceed the others by ~200 (log2
     # units): past the fast pass's headroom, so P' would overflow bf16. The fast pass flags the

@@ -1193,9 +1193,15 @@ constexpr int kMlaVB = 4;           // V fragments per pipelined batch (two read
 constexpr float kMlaSlack = 8.0f;   // log2-domain headroom of the lazily raised softmax max
 constexpr float kMlaHeadroom = 64.0f;  // log2-domain headroom of the fast pass's fixed reference
 // Balance units charged for the start of a sequence beside its steps: a workgroup whose range begins another
-// sequence pays for its query fragments, ring fill and partial again, about 7 steps' worth (128 sequences of
-// 512-4096 tokens, 128 heads: 143 us with steps alone, 126 / 124 / 127 us with 4 / 7 / 10).
-constexpr int kMlaSegCost = 7;
+// sequence pays for its query fragments, ring fill and partial again, about 7 steps' worth with 128 heads (128
+// sequences of 512-1500 tokens: 93 us with steps alone, 86 / 86 / 91 us with 4 / 7 / 10). With up to 64 heads
+// there is less to load and write, about 3 steps (the same with 16 heads: 64 us, then 65 / 70 / 73 us with 3 / 7 /
+// 10; with 64 heads 76, then 72 / 76 / 79 us). Up to 32 sequences the larger charge measured better there too (16
+// sequences of 500-2000 tokens, 16 heads: 49 us, then 44 / 41 us with 3 / 7; one of 200: 50, then 41 / 35, as the
+// merge walks past the ranges that hold no step).
+// (A template argument: read from the arguments it cost a single sequence 1.2 us.)
+constexpr int kMlaSegCost = 7, kMlaSegCostFewHeads = 3;
+inline bool mla_few_heads(int64_t b, int hq) { return hq <= 64 && b > 32; }
 constexpr int kMlaWgs = 256;         // workgroups of a launch (one per CU of an MI355X)
 
 struct MlaArgs {
@@ -1217,7 +1223,7 @@ struct MlaArgs {
   float* part_ml;  // [slots, kMlaHeads, 2]
   int32_t* flags;  // [slots, kMlaWaves]: 1 = that wave's heads need the rescaling pass
   int32_t* wgflags;  // [kMlaWgs, kMlaWaves]: 1 = some segment of that workgroup's wave was flagged
-  int64_t* steps;  // [0] = 32-token steps of all sequences S, [1 + b] = steps before sequence b
+  int64_t* steps;  // [0] = balance units of all sequences S, [1 + b] = units before sequence b
 };
 
 // Raw ring stage: [latent 32 x 512 B][rope 32 x 128 B][one 256 B scale slot per wave].
@@ -1641,18 +1647,19 @@ __device__ __forceinline__ void mla_segment(const MlaArgs& a, char* smem, bool& 
   }
 }
 
-// Balance units of a sequence: its 32-token steps, and kMlaSegCost for its start, the cost of one more segment
-// in a workgroup (query fragments, ring fill, partial).
-__device__ __forceinline__ int64_t mla_units(int64_t len) { return len > 0 ? (len + kMlaStep - 1) / kMlaStep + kMlaSegCost : 0; }
+// Balance units of sequence b: its 32-token steps, and SC for its start.
+template <int SC>
+__device__ __forceinline__ int64_t mla_units(const MlaArgs& a, int64_t b) {
+  const int64_t len = kv_len(a, b);
+  return len > 0 ? (len + kMlaStep - 1) / kMlaStep + SC : 0;
+}
 
 // The kMlaWgs workgroups of a launch split all 32-token steps (head group major, then sequence)
 // into equal contiguous ranges, so every CU gets the same work whatever the lengths; a workgroup
 // runs one segment per sequence its range touches. Workgroup 0 of the fast pass also records the
 // step prefix the merge uses to find a sequence's partials.
-template <int DN, int DR, bool RESCALE>
-__global__ __launch_bounds__(64 * kMlaWaves) __attribute__((amdgpu_waves_per_eu(1, 1)))
-void mla_decode_kernel(MlaArgs a) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+template <int DN, int DR, bool RESCALE, int SC>
+__device__ __forceinline__ void mla_decode_walk(const MlaArgs& a, char* smem) {
   const int lane = threadIdx.x & 63;
   const int64_t nb = a.b;
   const int64_t wg = blockIdx.x;
@@ -1663,14 +1670,14 @@ void mla_decode_kernel(MlaArgs a) {
   }
   bool ov_seen = false;
   int64_t mine = 0;
-  for (int64_t c = lane; c < nb; c += 64) mine += mla_units(kv_len(a, c));
+  for (int64_t c = lane; c < nb; c += 64) mine += mla_units<SC>(a, c);
   const int64_t S = uniform64(wave_sum64(mine));
   const int64_t W = S * a.hgroups;
   if (!RESCALE && wg == 0 && threadIdx.x < 64) {
     int64_t carry = 0;
     for (int64_t c = 0; c < nb; c += 64) {
       const int64_t i = c + lane;
-      const int64_t n = i < nb ? mla_units(kv_len(a, i)) : 0;
+      const int64_t n = i < nb ? mla_units<SC>(a, i) : 0;
       const int64_t incl = wave_incl_scan64(n, lane) + carry;
       if (i < nb) a.steps[1 + i] = incl - n;
       carry = __shfl(incl, 63, 64);
@@ -1689,7 +1696,7 @@ void mla_decode_kernel(MlaArgs a) {
     int64_t carry = 0;
     for (int64_t c = 0; c < nb; c += 64) {
       const int64_t i = c + lane;
-      const int64_t n = i < nb ? mla_units(kv_len(a, i)) : 0;
+      const int64_t n = i < nb ? mla_units<SC>(a, i) : 0;
       const int64_t incl = wave_incl_scan64(n, lane) + carry;
       const uint64_t hit = __ballot(i < nb && n > 0 && incl - n <= x && x < incl);
       if (hit) {
@@ -1705,11 +1712,11 @@ void mla_decode_kernel(MlaArgs a) {
   pb = uniform64(pb);
   for (int64_t g = g0; g < g1;) {
     const int64_t len = kv_len(a, b);
-    const int64_t n = mla_units(len);
+    const int64_t n = mla_units<SC>(a, b);
     const int64_t seg = min(g1 - g, pb + n - x);
-    // units [u0, u0 + seg) of the sequence; the first kMlaSegCost carry no tokens
+    // units [u0, u0 + seg) of the sequence; the first SC carry no tokens
     const int64_t u0 = x - pb;
-    const int64_t s0 = imax64(u0, kMlaSegCost) - kMlaSegCost, s1 = imax64(u0 + seg, kMlaSegCost) - kMlaSegCost;
+    const int64_t s0 = imax64(u0, SC) - SC, s1 = imax64(u0 + seg, SC) - SC;
     const int64_t slot = hg * (kMlaWgs + nb) + wg + b;
     bool run = s1 > s0;
     if constexpr (RESCALE) {
@@ -1723,10 +1730,25 @@ void mla_decode_kernel(MlaArgs a) {
       pb += n;
       do {
         if (++b == nb) { b = 0; pb = 0; x = 0; ++hg; }
-      } while (g < g1 && mla_units(kv_len(a, b)) == 0);
+      } while (g < g1 && mla_units<SC>(a, b) == 0);
     }
   }
   if (!RESCALE && lane == 0) *wgflag = ov_seen ? 1 : 0;
+}
+
+template <int DN, int DR, bool RESCALE>
+__global__ __launch_bounds__(64 * kMlaWaves) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void mla_decode_kernel(MlaArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  mla_decode_walk<DN, DR, RESCALE, kMlaSegCost>(a, smem);
+}
+
+// The same with the smaller charge for a sequence's start.
+template <int DN, int DR, bool RESCALE>
+__global__ __launch_bounds__(64 * kMlaWaves) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void mla_decode_few_heads_kernel(MlaArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  mla_decode_walk<DN, DR, RESCALE, kMlaSegCostFewHeads>(a, smem);
 }
 
 // Merge the partials of a sequence's heads: one wave per pair of heads (each lane owns 8
@@ -1735,7 +1757,7 @@ void mla_decode_kernel(MlaArgs a) {
 // (uniform across the wave), and every partial's O values are loaded before the weights that
 // scale them are known, so a wave waits on few dependent round trips.
 constexpr int kMlaCombineHeads = 8;  // heads per combine workgroup (2 per wave)
-template <int DN>
+template <int DN, int SC>
 __global__ __launch_bounds__(256) void mla_combine_kernel(MlaArgs a, uint16_t* out, float* lse) {
   static_assert(DN == 512, "one lane holds 8 of the 512 latent dims");
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -1744,7 +1766,7 @@ __global__ __launch_bounds__(256) void mla_combine_kernel(MlaArgs a, uint16_t* o
   const int h0 = static_cast<int>(blockIdx.x % per_b) * kMlaCombineHeads + 2 * wv;
   if (h0 >= a.hq) return;
   const bool two = h0 + 1 < a.hq;
-  const int64_t n = mla_units(kv_len(a, b));
+  const int64_t n = mla_units<SC>(a, b);
   uint4* o0 = reinterpret_cast<uint4*>(out + (b * a.hq + h0) * DN) + lane;
   uint4* o1 = reinterpret_cast<uint4*>(out + (b * a.hq + h0 + 1) * DN) + lane;
   if (n == 0) {
@@ -1755,7 +1777,7 @@ __global__ __launch_bounds__(256) void mla_combine_kernel(MlaArgs a, uint16_t* o
   }
   const int64_t S = a.steps[0], W = S * a.hgroups;
   const int hg = h0 / kMlaHeads, hl = h0 % kMlaHeads;  // h0 is even, so both heads share hg
-  const int64_t x0 = hg * S + a.steps[1 + b] + kMlaSegCost, x1 = x0 + n - kMlaSegCost;  // units of its steps
+  const int64_t x0 = hg * S + a.steps[1 + b] + SC, x1 = x0 + n - SC;  // units of its steps
   const int64_t w_first = ((x0 + 1) * kMlaWgs - 1) / W, w_last = (x1 * kMlaWgs - 1) / W;
   const int ns = static_cast<int>(w_last - w_first + 1);
   const int64_t row0 = (hg * (kMlaWgs + a.b) + w_first + b) * kMlaHeads + hl;  // partial s: row0 + s * kMlaHeads
@@ -2126,10 +2148,13 @@ extern "C" int tai_fia_mla_decode(const void* q_nope, const void* q_rope, const 
   // the LDS attribute is set once per process; a function-local static initialiser runs exactly
   // once even when several host threads reach it together
   static const bool lds_ok = [] {
-    const bool ok = hipFuncSetAttribute(reinterpret_cast<const void*>(&mla_decode_kernel<512, 64, false>),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, kMlaLds) == hipSuccess &&
-                    hipFuncSetAttribute(reinterpret_cast<const void*>(&mla_decode_kernel<512, 64, true>),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, kMlaLds) == hipSuccess;
+    auto set = [](const void* f) {
+      return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kMlaLds) == hipSuccess;
+    };
+    const bool ok = set(reinterpret_cast<const void*>(&mla_decode_kernel<512, 64, false>)) &&
+                    set(reinterpret_cast<const void*>(&mla_decode_kernel<512, 64, true>)) &&
+                    set(reinterpret_cast<const void*>(&mla_decode_few_heads_kernel<512, 64, false>)) &&
+                    set(reinterpret_cast<const void*>(&mla_decode_few_heads_kernel<512, 64, true>));
     (void)hipGetLastError();
     return ok;
   }();
@@ -2139,9 +2164,16 @@ extern "C" int tai_fia_mla_decode(const void* q_nope, const void* q_rope, const 
   }
   // fast pass, then the rescaling pass over the segments the fast pass flagged (it skips the others)
   const dim3 grid(kMlaWgs);
-  mla_decode_kernel<512, 64, false><<<grid, 64 * kMlaWaves, kMlaLds, st>>>(a);
-  mla_decode_kernel<512, 64, true><<<grid, 64 * kMlaWaves, kMlaLds, st>>>(a);
-  const int64_t combine_wgs = b * ((hq + kMlaCombineHeads - 1) / kMlaCombineHeads);
-  mla_combine_kernel<512><<<dim3(static_cast<unsigned>(combine_wgs)), 256, 0, st>>>(a, static_cast<uint16_t*>(out), lse);
+  const unsigned combine_wgs = static_cast<unsigned>(b * ((hq + kMlaCombineHeads - 1) / kMlaCombineHeads));
+  uint16_t* o = static_cast<uint16_t*>(out);
+  if (mla_few_heads(b, hq)) {
+    mla_decode_few_heads_kernel<512, 64, false><<<grid, 64 * kMlaWaves, kMlaLds, st>>>(a);
+    mla_decode_few_heads_kernel<512, 64, true><<<grid, 64 * kMlaWaves, kMlaLds, st>>>(a);
+    mla_combine_kernel<512, kMlaSegCostFewHeads><<<combine_wgs, 256, 0, st>>>(a, o, lse);
+  } else {
+    mla_decode_kernel<512, 64, false><<<grid, 64 * kMlaWaves, kMlaLds, st>>>(a);
+    mla_decode_kernel<512, 64, true><<<grid, 64 * kMlaWaves, kMlaLds, st>>>(a);
+    mla_combine_kernel<512, kMlaSegCost><<<combine_wgs, 256, 0, st>>>(a, o, lse);
+  }
   return launch_status("tai_fia_mla_decode");
 }
