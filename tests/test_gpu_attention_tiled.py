@@ -171,9 +171,12 @@ def _packed(monkeypatch, lq, lk, hq, hkv, d, bs, seed, dt=torch.bfloat16, layout
     ([130, 3], [130, 3000], 8, 8, 64, 32),                          # one head a group, a tile over two pages
     ([20, 33, 1], [900, 33, 4000], 64, 2, 64, 128),                 # 32 heads a group
     ([300, 1], [9, 1], 16, 2, 128, 64),                             # rows that see nothing
-    ([2, 0] * 35, [2 + 5 * i for i in range(70)], 8, 2, 64, 32),    # more sequences than the kernel plans by itself
-    ([512], [512], 16, 4, 128, 128),                                # the most rows it does, and one more
-    ([513], [700], 16, 4, 128, 128),
+    ([2, 0] * 35, [2 + 5 * i for i in range(70)], 8, 2, 64, 32),    # short sequences, every other one empty
+    ([512], [512], 16, 4, 128, 128),                                # the most rows that the kernel plans by itself,
+    ([513], [700], 16, 4, 128, 128),                                # and one more
+    ([1, 0, 2, 1] * 128, [(7 * i) % 90 for i in range(512)], 4, 2, 64, 32),        # the most sequences that it does,
+    ([1, 0, 2, 1] * 128 + [1], [(7 * i) % 90 for i in range(513)], 4, 2, 64, 32),  # and one more
+    ([300] + [1] * 15 + [280, 0, 1], [300] + [40] * 15 + [500, 9, 77], 16, 2, 64, 32),  # long ones in one planning wave
 ])
 @pytest.mark.parametrize("mode", [{"sparse_mode": 3}, {}, {"sparse_mode": 4, "pre_tokens": 70, "next_tokens": 9}])
 def test_packed_paged(monkeypatch, lq, lk, hq, hkv, d, bs, mode):

@@ -38,7 +38,8 @@ struct PackedArgs {
   float* part_ml;     // [2 * kKWgs][256][2]
   bool plan_here;     // few sequences of few blocks: the main kernel plans by itself
 };
-constexpr int kKPlanSeqs = 64, kKPlanBlocks = 8;
+constexpr int kKPlanSeqs = 512;  // the main kernel's threads
+constexpr int kKPlanBlocks = 8;
 
 struct SeqInfo {
   int64_t q_start, lq, lk, kv_base, off;
@@ -97,17 +98,34 @@ __device__ __forceinline__ int tiles_before(const Block& b, int64_t u) {
   return static_cast<int>((imax64(u, kKItem) - kKItem + b.unit - 1) / b.unit);
 }
 
+// Cost of sequence b's blocks, by one thread.
+__device__ __forceinline__ int64_t seq_cost(const PackedArgs& p, int64_t b) {
+  const SeqInfo s = seq_info(p, b);
+  const int n = seq_blocks(p, s);
+  int64_t c = 0;
+  for (int j = 0; j < n; ++j) c += block_cost(block_of(p, s, j));
+  return c;
+}
+
+// A lane per sequence, so that many short ones are planned at once (a wave each took 23 us for 256 single tokens, beside 39 of the main kernel);
+// a sequence of many blocks is summed by its whole wave. Neighbouring sequences go to different waves.
 __global__ __launch_bounds__(1024) void packed_plan_kernel(PackedArgs p) {
   __shared__ int64_t red[16];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  // a wave per sequence, lanes over its blocks
-  for (int64_t b = w; b < p.a.b; b += 16) {
-    const SeqInfo s = seq_info(p, b);
-    const int n = seq_blocks(p, s);
-    int64_t c = 0;
-    for (int j = lane; j < n; j += 64) c += block_cost(block_of(p, s, j));
-    c = wave_sum64(c) * p.a.hkv;
-    if (lane == 0) p.pref[b + 1] = c;
+  for (int64_t b0 = 0; b0 < p.a.b; b0 += 1024) {
+    const int64_t b = b0 + 16 * lane + w;
+    const bool wide = b < p.a.b && seq_blocks(p, seq_info(p, b)) > kKPlanBlocks;
+    int64_t c = b < p.a.b && !wide ? seq_cost(p, b) : 0;
+    for (uint64_t todo = __ballot(wide); todo; todo &= todo - 1) {
+      const int k = __ffsll(static_cast<unsigned long long>(todo)) - 1;
+      const SeqInfo s = seq_info(p, b0 + 16 * k + w);
+      const int n = seq_blocks(p, s);
+      int64_t x = 0;
+      for (int j = lane; j < n; j += 64) x += block_cost(block_of(p, s, j));
+      x = wave_sum64(x);
+      if (lane == k) c = x;
+    }
+    if (b < p.a.b) p.pref[b + 1] = c * p.a.hkv;
   }
   __threadfence_block();
   __syncthreads();
@@ -480,23 +498,21 @@ template <int D, bool F16>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void packed_kernel(PackedArgs p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   __shared__ int64_t s_pref[kKPlanSeqs + 1];
+  __shared__ int64_t red[16];
   const int lane = threadIdx.x & 63;
   const int64_t* pref = p.pref;
   if (p.plan_here) {
-    // a lane per sequence; the plan kernel and its launch cost small calls more (4 tokens over 64: 15.8 us with it, 13.1 without)
-    if (threadIdx.x < 64) {
-      int64_t c = 0;
-      if (lane < p.a.b) {
-        const SeqInfo s = seq_info(p, lane);
-        const int n = seq_blocks(p, s);
-        for (int j = 0; j < n; ++j) c += block_cost(block_of(p, s, j));
-      }
-      const int64_t incl = wave_incl_scan64(c * p.a.hkv, lane);
-      s_pref[lane + 1] = incl;
-      if (lane == 0) s_pref[0] = 0;
+    // a thread per sequence; the plan kernel and its launch cost small calls more (4 tokens over 64: 15.8 us with it,
+    // 13.1 without; 256 single tokens over 64, 16 / 8 heads of 64: 64 and 41 us). Up to 64 sequences one wave does it, which saves the others'
+    // part of the scan, 0.4 us.
+    if (p.a.b > 64 || threadIdx.x < 64) {
+      const int64_t c = threadIdx.x < p.a.b ? seq_cost(p, threadIdx.x) * p.a.hkv : 0;
+      const int64_t incl = p.a.b > 64 ? block_incl_scan<false>(c, red) : wave_incl_scan64(c, lane);
+      s_pref[threadIdx.x + 1] = incl;
+      if (threadIdx.x == 0) s_pref[0] = 0;
       if (blockIdx.x == 0) {  // for the merge
-        if (lane < p.a.b) p.pref[lane + 1] = incl;
-        if (lane == 0) p.pref[0] = 0;
+        if (threadIdx.x < p.a.b) p.pref[threadIdx.x + 1] = incl;
+        if (threadIdx.x == 0) p.pref[0] = 0;
       }
     }
     __syncthreads();
