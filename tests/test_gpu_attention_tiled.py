@@ -202,6 +202,13 @@ def test_packed_scales_and_rising_logits(monkeypatch, dt, scale):
                           sparse_mode=3), 4.5)
 
 
+def test_packed_nan_scale(monkeypatch):
+    """A scale of NaN gives NaN wherever a row sees a key, as in the general kernel."""
+    tiled, general = _packed(monkeypatch, [5, 0, 1], [70, 9, 300], 8, 2, 64, 64, 321, scale=math.nan, sparse_mode=3)
+    assert torch.isnan(general[0]).all() and torch.isnan(tiled[0]).all()
+    assert torch.equal(tiled[1], general[1])
+
+
 def test_packed_sink(monkeypatch):
     sink = torch.linspace(-3, 6, 16)
     sink[5] = -math.inf

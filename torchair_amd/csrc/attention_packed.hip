@@ -710,7 +710,9 @@ int packed_run(const tai_fia_general_args& a, void* workspace, size_t ws_bytes, 
   p.g = a.hq / a.hkv;
   p.kv_cap = a.block_table ? a.max_blocks * a.block_size : a.s_kv;
   // a zero scale makes every score zero, which the smallest normal scale gives up to rounding far below the output's
-  p.scale_log2 = fmaxf(fabsf(a.scale) * kLog2e, 1.17549435e-38f);
+  // (written so that a NaN stays one)
+  p.scale_log2 = fabsf(a.scale) * kLog2e;
+  if (p.scale_log2 < 1.17549435e-38f) p.scale_log2 = 1.17549435e-38f;
   p.neg_scale = a.scale < 0.0f;
   char* ws = static_cast<char*>(workspace);
   p.pref = reinterpret_cast<int64_t*>(ws);
