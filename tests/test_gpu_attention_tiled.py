@@ -304,3 +304,47 @@ def test_packed_band_does_not_read_released_pages(bs, dt):
     want, got = call(bt), call(gone)
     assert np.isfinite(want[0].float().cpu().numpy()).all()
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+def _guarded(monkeypatch, call):
+    """(call's result, workspace bytes) with 1 MB of a pattern behind the workspace, which must stay as it was."""
+    real, seen = _lib.call, []
+
+    def spy(name, *args):
+        if name != "tai_fia_tiled":
+            return real(name, *args)
+        a, _, n, stream = args
+        buf = torch.full((n + (1 << 20),), 0x5A, dtype=torch.uint8, device=DEV)
+        real(name, a, buf.data_ptr(), n, stream)
+        assert bool((buf[n:] == 0x5A).all()), "written past the workspace"
+        seen.append(n)
+
+    monkeypatch.setattr(_fia._lib, "call", spy)
+    out = call()
+    monkeypatch.setattr(_fia._lib, "call", real)
+    assert len(seen) == 1
+    return out, seen[0]
+
+
+@pytest.mark.parametrize("lq,lk,hq,hkv,d,bs,most", [
+    ([1], [1], 4, 4, 64, 32, 1 << 18),
+    ([1] * 4, [128, 7, 64, 128], 32, 8, 128, 128, 1 << 21),
+    ([3, 0, 9], [500, 4, 9], 16, 2, 128, 64, 1 << 24),
+    ([30] * 3, [200, 30, 77], 8, 8, 64, 32, 1 << 23),                  # one wave of columns a block
+    ([40] * 3, [200, 40, 77], 16, 4, 128, 32, 1 << 25),                # five
+    ([200, 1, 60], [3000, 2000, 60], 32, 8, 128, 128, 66 << 20),        # 256 ranges of 256 columns
+])
+def test_packed_workspace_follows_the_call(monkeypatch, lq, lk, hq, hkv, d, bs, most):
+    """Small calls take a small workspace and stay inside it, and equal the general kernel."""
+    g = torch.Generator().manual_seed(380 + hq + len(lq))
+    bt, n = _table(lk, bs, g)
+    k, v = _kv(n, bs, hkv, d, torch.bfloat16, g)
+    q = torch.randn(sum(lq) + 2, hq, d, generator=g).to(torch.bfloat16).to(DEV)
+    print("case", lq, lk, hq, hkv, d, bs, flush=True)
+    call = lambda: FIA(q, k, v, actual_seq_lengths=torch.tensor(np.cumsum(lq), device=DEV),  # noqa: E731
+                       actual_seq_lengths_kv=torch.tensor(lk, device=DEV), block_table=bt.to(DEV), num_heads=hq,
+                       num_key_value_heads=hkv, input_layout="TND", block_size=bs, scale=d ** -0.5, sparse_mode=3,
+                       softmax_lse_flag=True)
+    got, size = _guarded(monkeypatch, call)
+    assert size <= most
+    _assert_same(got, _both(monkeypatch, call)[1], 4.5)

@@ -20,7 +20,7 @@
 namespace tai {
 namespace {
 
-constexpr int kKWgs = 256;       // ranges: one workgroup per CU
+constexpr int kKWgs = 256;       // most ranges: one workgroup per CU
 constexpr int kKCols = 256;      // columns per item
 // Cost of an item: kKItem units for its start (query load, ring fill, output) and per tile 2 units with up to
 // one wave per SIMD, 3 with two.
@@ -34,8 +34,10 @@ struct PackedArgs {
   int neg_scale;      // the scale is negative: Q is negated on load
   int64_t* pref;      // [b + 1] cost of the sequences before
   int4* rec;          // [ranges] the item each range leaves unfinished: {b, kv head, block, last range} (last = 0: none)
-  float* part_o;      // [2 * kKWgs][8 waves][D / 32][4][64 lanes][4]; slot 2r: the item range r continues, 2r + 1: leaves
-  float* part_ml;     // [2 * kKWgs][256][2]
+  int cap;            // most ranges this call can have
+  int waves;          // waves of a workgroup that can hold columns: 32 each of a block's at most 256
+  float* part_o;      // [2 * cap][waves][D / 32][4][64 lanes][4]; slot 2r: the item range r continues, 2r + 1: leaves
+  float* part_ml;     // [2 * cap][32 * waves][2]
   bool plan_here;     // few sequences of few blocks: the main kernel plans by itself
 };
 constexpr int kKPlanSeqs = 512;  // the main kernel's threads
@@ -422,8 +424,8 @@ __device__ __forceinline__ void packed_segment(const PackedArgs& p, char* smem, 
   }
   if (!wave_ok) return;
   l_run += __shfl_xor(l_run, 32, 64);
-  float* po = p.part_o + (static_cast<int64_t>(slot) * 8 + w) * 32 * D;
-  float* ml = p.part_ml + (static_cast<int64_t>(slot) * kKCols + 32 * w) * 2;
+  float* po = p.part_o + (static_cast<int64_t>(slot) * p.waves + w) * 32 * D;
+  float* ml = p.part_ml + (static_cast<int64_t>(slot) * p.waves + w) * 32 * 2;
   const int64_t out_off = q_offset(p, a.out_strides, s, b, row, head);
   uint16_t* op = static_cast<uint16_t*>(a.out);
   float* lse = nullptr;
@@ -490,7 +492,7 @@ __device__ __forceinline__ void packed_segment(const PackedArgs& p, char* smem, 
 
 // Ranges of a launch of W units: at least 6 units each, so that every range inside an item holds a tile's first
 // unit (a partial exists for each of them) and no workgroup starts for less than two tiles.
-__device__ __forceinline__ int64_t ranges_of(int64_t W) { return imax64(W > 0 ? 1 : 0, imin64(kKWgs, W / 6)); }
+__device__ __forceinline__ int64_t ranges_of(const PackedArgs& p, int64_t W) { return imax64(W > 0 ? 1 : 0, imin64(p.cap, W / 6)); }
 // The range a unit x of the launch's W belongs to, of R equal ones.
 __device__ __forceinline__ int64_t range_of(int64_t x, int64_t W, int64_t R) { return ((x + 1) * R - 1) / W; }
 
@@ -519,7 +521,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     pref = s_pref;
   }
   // consecutive ranges, which share a kv head's tiles, run on one XCD
-  const int64_t W = uniform64(pref[p.a.b]), R = ranges_of(W), per = (R + 7) / 8;
+  const int64_t W = uniform64(pref[p.a.b]), R = ranges_of(p, W), per = (R + 7) / 8;
   const int64_t r = (blockIdx.x % 8) * per + blockIdx.x / 8;
   if (blockIdx.x / 8 >= per || r >= R) return;
   const int64_t u0 = uniform64(r * W / R), u1 = uniform64((r + 1) * W / R);
@@ -587,17 +589,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   if (threadIdx.x == 0) p.rec[r] = rec;
 }
 
-// Blocks 0 .. 8 * kKWgs - 1: 32 columns (wave w) of the item range r leaves unfinished, over its partials. The
+// Blocks 0 .. waves * cap - 1: 32 columns (wave w) of the item range r leaves unfinished, over its partials. The
 // blocks after them write the rows that belong to no sequence (64 rows each).
 template <int D, bool F16>
 __global__ __launch_bounds__(256) void packed_merge_kernel(PackedArgs p) {
   using H = Half<F16>;
   const tai_fia_general_args& a = p.a;
   const int tid = threadIdx.x, lane = tid & 63;
-  if (blockIdx.x >= 8 * kKWgs) {
+  const uint32_t joins = static_cast<uint32_t>(p.waves) * p.cap;
+  if (blockIdx.x >= joins) {
     // a lane looks at each of the 64 rows (one after another they took 5 us where all belonged to a sequence: 64
     // single tokens over 500 keys, 16 / 8 heads of 64, 42.1 us then, 36.8 now)
-    const int64_t rows = a.q_cum ? a.s_q : a.b * a.s_q, v0 = (static_cast<int64_t>(blockIdx.x) - 8 * kKWgs) * 64;
+    const int64_t rows = a.q_cum ? a.s_q : a.b * a.s_q, v0 = static_cast<int64_t>(blockIdx.x - joins) * 64;
     const int64_t vl = v0 + lane, bl = a.q_cum ? 0 : vl / a.s_q;
     const bool spare = vl < rows && (a.q_cum ? vl >= a.q_cum[a.b - 1] : a.seq_lens_q && vl - bl * a.s_q >= a.seq_lens_q[bl]);
     for (uint64_t todo = __ballot(spare); todo; todo &= todo - 1) {
@@ -613,8 +616,8 @@ __global__ __launch_bounds__(256) void packed_merge_kernel(PackedArgs p) {
     }
     return;
   }
-  const int r = blockIdx.x >> 3, w = blockIdx.x & 7;
-  if (r >= ranges_of(p.pref[a.b])) return;
+  const int r = static_cast<int>(blockIdx.x / static_cast<uint32_t>(p.waves)), w = static_cast<int>(blockIdx.x) - r * p.waves;
+  if (r >= ranges_of(p, p.pref[a.b])) return;
   const int4 rec = p.rec[r];
   if (rec.w == 0) return;
   const SeqInfo s = seq_info(p, rec.x);
@@ -628,11 +631,11 @@ __global__ __launch_bounds__(256) void packed_merge_kernel(PackedArgs p) {
 #pragma unroll 2
   for (int q = r; q <= rec.w; ++q) {
     const int64_t slot = 2 * q + (q == r ? 1 : 0);
-    const float* po = p.part_o + (slot * 8 + w) * 32 * D;
+    const float* po = p.part_o + (slot * p.waves + w) * 32 * D;
     f32x4 v[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) v[e] = *reinterpret_cast<const f32x4*>(po + ((4 * e + (tid >> 6)) * 64 + lane) * 4);
-    const float2 st = *reinterpret_cast<const float2*>(p.part_ml + (slot * kKCols + 32 * w + (lane & 31)) * 2);
+    const float2 st = *reinterpret_cast<const float2*>(p.part_ml + ((slot * p.waves + w) * 32 + (lane & 31)) * 2);
     const float mn = fmaxf(m, st.x);
     const float c0 = m == -INFINITY ? 0.0f : exp2f(m - mn), c1 = st.x == -INFINITY ? 0.0f : exp2f(st.x - mn);
     l = l * c0 + st.y * c1;
@@ -663,15 +666,30 @@ __global__ __launch_bounds__(256) void packed_merge_kernel(PackedArgs p) {
         live ? (m + log2f(l)) * kLn2 : -INFINITY;
 }
 
+// What the call can have at most, from what the host knows of it. A range has at least 6 units, so small calls have
+// few ranges, and few rows fill few waves: the partials take 2 MB for 4 tokens over pages of 128 keys where 256
+// ranges of 256 columns take 64 MB.
+int packed_waves(const tai_fia_general_args& a) {
+  return static_cast<int>(cdiv(imin64(a.s_q * (a.hq / a.hkv), kKCols), 32));
+}
+int packed_cap(const tai_fia_general_args& a) {
+  const int64_t blocks = cdiv(a.s_q * (a.hq / a.hkv), kKCols);  // of a sequence; packed ones share them, each with a rest
+  const int64_t items = a.hkv * (a.q_cum ? blocks + a.b : blocks * a.b);
+  if (items >= 2 * kKWgs) return kKWgs;
+  const int64_t tiles = cdiv(a.block_table ? a.max_blocks * a.block_size : a.s_kv, kPKV);
+  return static_cast<int>(imax64(1, imin64(kKWgs, items * (kKItem + tiles * (packed_waves(a) > 4 ? 3 : 2)) / 6)));
+}
+
 struct PackedWs {
   size_t rec, part_o, part_ml, total;
 };
 PackedWs packed_ws(const tai_fia_general_args& a) {
+  const size_t waves = 2 * static_cast<size_t>(packed_cap(a)) * packed_waves(a);
   PackedWs w;
   w.rec = (static_cast<size_t>(a.b + 1) * sizeof(int64_t) + 255) / 256 * 256;
-  w.part_o = w.rec + kKWgs * sizeof(int4);
-  w.part_ml = w.part_o + static_cast<size_t>(2 * kKWgs) * kKCols * a.dv * sizeof(float);
-  w.total = w.part_ml + static_cast<size_t>(2 * kKWgs) * kKCols * 2 * sizeof(float);
+  w.part_o = (w.rec + packed_cap(a) * sizeof(int4) + 255) / 256 * 256;
+  w.part_ml = w.part_o + waves * 32 * a.dv * sizeof(float);
+  w.total = w.part_ml + waves * 32 * 2 * sizeof(float);
   return w;
 }
 
@@ -708,6 +726,8 @@ int packed_run(const tai_fia_general_args& a, void* workspace, size_t ws_bytes, 
   p.a.pre_tokens = imin64(imax64(a.pre_tokens, -kNoBound), kNoBound);
   p.a.next_tokens = imin64(imax64(a.next_tokens, -kNoBound), kNoBound);
   p.g = a.hq / a.hkv;
+  p.cap = packed_cap(a);
+  p.waves = packed_waves(a);
   p.kv_cap = a.block_table ? a.max_blocks * a.block_size : a.s_kv;
   // a zero scale makes every score zero, which the smallest normal scale gives up to rounding far below the output's
   // (written so that a NaN stays one)
@@ -737,14 +757,15 @@ int packed_run(const tai_fia_general_args& a, void* workspace, size_t ws_bytes, 
   p.plan_here = a.b <= kKPlanSeqs && cdiv(a.s_q * p.g, kKCols) <= kKPlanBlocks;
   if (!p.plan_here) packed_plan_kernel<<<1, 1024, 0, st>>>(p);
   const int64_t rows = a.q_cum ? a.s_q : a.b * a.s_q;
-  const unsigned mgrid = static_cast<unsigned>(8 * kKWgs + cdiv(rows, 64));
+  const unsigned mgrid = static_cast<unsigned>(p.waves * p.cap + cdiv(rows, 64));
+  const unsigned grid = static_cast<unsigned>(8 * cdiv(p.cap, 8));
   auto launch = [&](auto f16c) {
     constexpr bool F16 = decltype(f16c)::value;
     if (a.dk1 == 64) {
-      packed_kernel<64, F16><<<kKWgs, 512, PrefillTile<64>::kLds, st>>>(p);
+      packed_kernel<64, F16><<<grid, 512, PrefillTile<64>::kLds, st>>>(p);
       packed_merge_kernel<64, F16><<<mgrid, 256, 0, st>>>(p);
     } else {
-      packed_kernel<128, F16><<<kKWgs, 512, PrefillTile<128>::kLds, st>>>(p);
+      packed_kernel<128, F16><<<grid, 512, PrefillTile<128>::kLds, st>>>(p);
       packed_merge_kernel<128, F16><<<mgrid, 256, 0, st>>>(p);
     }
   };
