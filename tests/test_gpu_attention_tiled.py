@@ -348,3 +348,18 @@ def test_packed_workspace_follows_the_call(monkeypatch, lq, lk, hq, hkv, d, bs, 
     got, size = _guarded(monkeypatch, call)
     assert size <= most
     _assert_same(got, _both(monkeypatch, call)[1], 4.5)
+
+
+@pytest.mark.parametrize("lens,hq,sq,bs,most", [
+    ([1], 16, 1, 32, 1 << 20),
+    ([128], 128, 1, 128, 6 << 20),
+    ([64, 0, 3], 40, 2, 32, 6 << 20),
+    ([100, 31], 136, 1, 32, 23 << 20),
+    ([4000] * 3, 128, 1, 128, 129 << 20),  # 256 ranges of 128 heads
+])
+def test_mla_rows_workspace_follows_the_call(monkeypatch, lens, hq, sq, bs, most):
+    call = _mla_call(_mla(lens, hq, sq, bs, 390 + hq), lens, hq, bs)
+    print("case", lens, hq, sq, bs, flush=True)
+    got, size = _guarded(monkeypatch, call)
+    assert size <= most
+    _assert_same(got, _both(monkeypatch, call)[1], 4.0)

@@ -63,7 +63,7 @@ __device__ __forceinline__ RowInfo row_info(const tai_fia_general_args& a, int64
 // SIMD: 36 score, 64 P.V) because its score, softmax and P.V phases follow one another between the barriers;
 // a segment costs about 25 us on top (query fragments, ring fill, 256 KB of partial per workgroup).
 constexpr int kRStep = 32;
-constexpr int kRWgs = 256;    // one workgroup per CU
+constexpr int kRWgs = 256;    // at most: one workgroup per CU
 constexpr int kRHeads = 128;
 constexpr int kRRing = 3;
 constexpr int kRRope = kRStep * 1024;            // rope rows behind the latent rows of a stage
@@ -80,8 +80,8 @@ struct MlaRowsArgs {
   int64_t nv;     // query rows
   int hgroups, hcap;
   int64_t* pref;  // [nv + 1] balance units before each row
-  float* part_o;  // [2 * kRWgs][hcap][512]: slot 2w of the row range w continues, 2w + 1 of the row it leaves unfinished
-  float* part_ml; // [2 * kRWgs][hcap][2]
+  float* part_o;  // [2 * ranges][hcap][512]: slot 2w of the row range w continues, 2w + 1 of the row it leaves unfinished
+  float* part_ml; // [2 * ranges][hcap][2]
   float scale_log2;
   bool pref_ready;
 };
@@ -542,19 +542,33 @@ __global__ __launch_bounds__(256) void mla_rows_merge_kernel(MlaRowsArgs g) {
   if (wv == 0 && lane == 0) store_lse(a, qb, qt, head, live ? (M + log2f(L)) * kLn2 : -INFINITY);
 }
 
+int64_t query_rows(const tai_fia_general_args& a) { return a.q_cum ? a.s_q : a.b * a.s_q; }
+
+// A workgroup whose range begins another row loads query fragments, fills the ring and writes a partial again:
+// about 7 steps' worth with 128 heads (32 sequences of 512-4096 tokens: 85 us with steps alone, 75 / 65 / 67 us
+// with 4 / 7 / 10), less with few heads (100 sequences, 16 heads: 61, then 58 / 60 / 65 us).
+int mla_rows_seg_cost(int64_t hq) { return hq > 64 ? 7 : 4; }
+
+// The most ranges the call can have: one per unit, from the rows and the keys a block-table row can hold (no row is
+// longer, see row_info). One sequence of up to 128 keys takes 6 MB of partials, not 128.
+int mla_rows_cap(const tai_fia_general_args& a) {
+  const int64_t rows = query_rows(a) * cdiv(a.hq, kRHeads);
+  if (rows >= kRWgs || a.max_blocks >= kRWgs) return kRWgs;
+  const int64_t steps = imin64(a.block_size / kRStep, kRWgs) * a.max_blocks;
+  return static_cast<int>(imin64(kRWgs, rows * (steps + mla_rows_seg_cost(a.hq))));
+}
+
 struct MlaRowsWs {
   size_t part_o, part_ml, total;
 };
-MlaRowsWs mla_rows_ws(int64_t nv, int64_t hq) {
-  const size_t hcap = static_cast<size_t>(imin64(hq, kRHeads));
+MlaRowsWs mla_rows_ws(const tai_fia_general_args& a) {
+  const size_t heads = 2 * static_cast<size_t>(mla_rows_cap(a)) * static_cast<size_t>(imin64(a.hq, kRHeads));
   MlaRowsWs w;
-  w.part_o = (static_cast<size_t>(nv + 1) * sizeof(int64_t) + 255) / 256 * 256;
-  w.part_ml = w.part_o + 2 * kRWgs * hcap * 512 * sizeof(float);
-  w.total = w.part_ml + 2 * kRWgs * hcap * 2 * sizeof(float);
+  w.part_o = (static_cast<size_t>(query_rows(a) + 1) * sizeof(int64_t) + 255) / 256 * 256;
+  w.part_ml = w.part_o + heads * 512 * sizeof(float);
+  w.total = w.part_ml + heads * 2 * sizeof(float);
   return w;
 }
-
-int64_t query_rows(const tai_fia_general_args& a) { return a.q_cum ? a.s_q : a.b * a.s_q; }
 
 // 32 rows of a tile stay below 2^31 bytes
 bool small_row(int64_t stride) { return stride >= 0 && stride < (int64_t(1) << 24); }
@@ -579,7 +593,7 @@ int mla_rows(const tai_fia_general_args& a, void* workspace, size_t ws_bytes, hi
   g.a = a;
   g.a.next_tokens = imin64(imax64(a.next_tokens, -kNoBound), kNoBound);
   g.nv = query_rows(a);
-  const MlaRowsWs w = mla_rows_ws(g.nv, a.hq);
+  const MlaRowsWs w = mla_rows_ws(a);
   if (workspace == nullptr || ws_bytes < w.total) {
     set_error("tai_fia_tiled: workspace of %zu bytes, need %zu", ws_bytes, w.total);
     return TAI_ERR_WORKSPACE;
@@ -608,13 +622,10 @@ int mla_rows(const tai_fia_general_args& a, void* workspace, size_t ws_bytes, hi
   auto launch = [&](auto sc) {
     constexpr int SC = decltype(sc)::value;
     if (g.pref_ready) mla_rows_prefix_kernel<SC><<<1, 1024, 0, st>>>(g);
-    mla_rows_kernel<SC><<<kRWgs, 512, kRLds, st>>>(g);
+    mla_rows_kernel<SC><<<mla_rows_cap(a), 512, kRLds, st>>>(g);
     mla_rows_merge_kernel<SC><<<static_cast<unsigned>(g.nv * a.hq), 256, 0, st>>>(g);
   };
-  // A workgroup whose range begins another row loads query fragments, fills the ring and writes a partial again:
-  // about 7 steps' worth with 128 heads (32 sequences of 512-4096 tokens: 85 us with steps alone, 75 / 65 / 67 us
-  // with 4 / 7 / 10), less with few heads (100 sequences, 16 heads: 61, then 58 / 60 / 65 us).
-    if (a.hq > 64) launch(std::integral_constant<int, 7>());
+  if (mla_rows_seg_cost(a.hq) == 7) launch(std::integral_constant<int, 7>());
   else launch(std::integral_constant<int, 4>());
   return launch_status("tai_fia_tiled");
 }
@@ -626,7 +637,7 @@ using namespace tai;
 
 extern "C" size_t tai_fia_tiled_workspace_size(const tai_fia_general_args* args) {
   if (!args) return 0;
-  if (mla_rows_takes(*args)) return mla_rows_ws(query_rows(*args), args->hq).total;
+  if (mla_rows_takes(*args)) return mla_rows_ws(*args).total;
   return packed_takes(*args) ? packed_workspace(*args) : 0;
 }
 
