@@ -437,7 +437,7 @@ int tai_fia_paged_decode_sink(const void* q, const void* k_cache, const void* v_
 /* The same over int8 key / value caches with per-channel antiquant scales and no offsets
  * (key_antiquant_scale / value_antiquant_scale, mode 0; prototype experiment_ops.h:3922-3932):
  * k = k_cache * k_scale[h * d + c], v = v_cache * v_scale[h * d + c] (fp32, [hkv * d]). The bytes become fp16
- * MFMA operands in registers; the query takes the key scale (rounded to fp16, scaled per head) and the merge
+ * MFMA operands in registers; the query takes the key scale (as two fp16 parts, scaled per head) and the merge
  * the value scale. Caches are int8 with byte strides (multiples of 8; 16-byte rows load faster). */
 size_t tai_fia_paged_decode_kv8_workspace_size(int64_t b, int hq, int hkv, int d, int64_t max_blocks,
                                                int block_size);

@@ -2,9 +2,10 @@
 integers: head dims, group sizes, both 16-bit query types, caches that start on 8 bytes only, sequences around
 the 32-token step and over many ranges, scores that rise along the keys, and queries far from 1.
 
-Bound: the query times the key scale is rounded to fp16 (2^-12 of each product) and P to fp16 (2^-12 of each
-term), the output to its type: |o - w| <= u |w| + (2^-11 + 2 d) max|v|, u = 2^-8 (bf16) or 2^-11 (fp16) and
-d = 2^-12 scale max_j sum|q ks k_j|, the largest error of a score."""
+Bound: the query times the key scale has 22 bits, P is rounded to fp16 (2^-12 of each term) and the output to its
+type. The first tests allow a query rounded once to fp16 (2^-12 of each product): |o - w| <= u |w| + (2^-11 + 2 d)
+max|v|, u = 2^-8 (bf16) or 2^-11 (fp16) and d = 2^-12 scale max_j sum|q ks k_j|, the largest error of a score; the
+last one takes d = 2^-20 scale max_j sum|q ks k_j|, 22 bits and sums in fp32."""
 import math
 
 import numpy as np
@@ -82,3 +83,35 @@ def test_int8_decode_query_ranges_and_rising_scores(qstd):
     """Queries whose products lie far outside fp16, and keys whose scores rise page by page."""
     _case(128, 8, 2, torch.bfloat16, 32, [500, 90], 420, qstd=qstd if qstd < 100 else 3.0, ramp=True)
     _case(64, 4, 1, torch.bfloat16, 64, [77], 421, qstd=qstd)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("mean,std,ints", [(0.0, 3.0, 32), (4.0, 0.1, 32), (4.0, 0.1, 1)])
+def test_int8_decode_scores_keep_their_precision(d, dt, mean, std, ints):
+    """Large scores, queries of one sign and keys of few steps, where a rounded query or sums far above the scores
+    would show: the lse within 2^-11 (the row sum takes the rounded P) and the scores' own 2^-20."""
+    g = torch.Generator(device=DEV).manual_seed(430 + d)
+    b, n, bs, hq, hkv = 4, 700, 64, 8, 2
+    nb = -(-n // bs)
+    bt = torch.arange(b * nb, device=DEV, dtype=torch.int32).view(b, nb)
+    q = (torch.randn(b, 1, hq * d, generator=g, device=DEV) * std + mean).to(dt)
+    k, v = [(torch.randn(b * nb, bs, hkv * d, generator=g, device=DEV) * ints).round().clamp(-127, 127).to(torch.int8)
+            for _ in range(2)]
+    ks, vs = [(torch.rand(hkv * d, generator=g, device=DEV) * 0.03 + 0.01) * 32 / ints for _ in range(2)]
+    print("case", d, dt, mean, std, ints, flush=True)
+    out, lse = FIA(q, k, v, actual_seq_lengths_kv=torch.tensor([n] * b, device=DEV), block_table=bt, num_heads=hq,
+                   num_key_value_heads=hkv, input_layout="BSH", block_size=bs, scale=d ** -0.5, key_antiquant_scale=ks,
+                   value_antiquant_scale=vs, softmax_lse_flag=True)
+    u = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11
+    k, v = [(x.double() * y.double()).cpu().numpy().reshape(b, nb * bs, hkv, d)[:, :n] for x, y in ((k, ks), (v, vs))]
+    q, out, lse = q.double().cpu().numpy().reshape(b, hq, d), out.double().cpu().numpy().reshape(b, hq, d), lse.cpu().numpy()
+    for i in range(b):
+        for h in range(hq):
+            kh, vh = k[i, :, h // (hq // hkv)], v[i, :, h // (hq // hkv)]
+            s = kh @ q[i, h] * d ** -0.5
+            err = 2.0 ** -20 * d ** -0.5 * (np.abs(kh) @ np.abs(q[i, h])).max()
+            p = np.exp(s - s.max())
+            w = p @ vh / p.sum()
+            assert (np.abs(out[i, h] - w) <= u * np.abs(w) + (2.0 ** -11 + 2 * err) * np.abs(vh).max()).all(), (i, h)
+            assert abs(lse.reshape(b, hq)[i, h] - (s.max() + np.log(p.sum()))) <= 2.0 ** -11 + err

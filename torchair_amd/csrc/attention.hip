@@ -332,17 +332,19 @@ void paged_decode_kernel(DecodeArgs a) {
 // ---------------------------------------------------------------------------- int8 caches
 // The same walk over int8 K/V with per-channel scales and no offsets: S = (q * key scale) . k8, and the merge
 // multiplies O by the value scale. A byte becomes a 16-bit operand without a conversion instruction: b ^ 0x80
-// under an fp16 exponent of 2^10 is 1152 + b, exactly. For K the 1152 stays in the product and leaves with
-// the score's one fused multiply-add (q.k + 1152 sum(q)); for V it is subtracted in packed fp16. So both MFMAs
-// take fp16, whatever the query's type: q * key scale is scaled to [1, 2) per head by a power of two and
-// rounded to fp16's 11 bits (the query's own type has 8 or 11), and P is kept 2^8 above 1 so that fp16's
-// smallest step lies 2^-32 below the row's largest term; the row sum takes the rounded P.
+// under an fp16 exponent of 2^10 is 1152 + b, exactly, and 1152 is subtracted in packed fp16. So both MFMAs take
+// fp16, whatever the query's type: q * key scale, scaled to [1, 2) per head by a power of two, enters as its fp16
+// rounding and the rest (times 2^11, into sums of its own), 22 bits in all, and P is kept 2^8 above 1 so that
+// fp16's smallest step lies 2^-32 below the row's largest term; the row sum takes the rounded P.
+// Error against 64 bits (700 keys, 32 / 8 heads of 128, fp16): 2.9e-4 of a row; with the query rounded once 3.4e-4 here
+// and 3.2e-4 on the 16-bit kernel, and with 1152 left in the keys' products, to be subtracted from the scores, up to
+// 1.5e-3 for queries of one sign over keys of one or two steps.
 //
-// The cache is read once, at one byte an element. The loop is bound by the conversions (about 130 of 170 vector
-// instructions per 32-token step and wave at D = 128), so two waves share a SIMD where the bf16 kernel runs one,
-// the max is raised lazily (no cross-lane reduction in a step) and the row sum reduced at the end.
-// Measured (64 sequences of 512-4096 tokens, 32 / 8 heads of 128): 60 us (this kernel 48, the merge 6) against
-// 318 us for widening the covered pages to 16 bits (212 us, 5 bytes moved per cache byte) before the 16-bit kernel.
+// The cache is read once, at one byte an element. Most of a step's vector instructions are conversions (160 of about
+// 200 at D = 128), so two waves share a SIMD where the bf16 kernel runs one, the max is raised lazily (no cross-lane
+// reduction in a step) and the row sum reduced at the end.
+// Measured (64 sequences of 512-4096 tokens, 32 / 8 heads of 128): 58 us (this kernel 46, the merge 5) against 318 us
+// for widening the covered pages to 16 bits (212 us, 5 bytes moved per cache byte) before the 16-bit kernel.
 template <int D>
 struct Decode8Tile {
   static constexpr int kCpr = D / 16;                 // 16-byte chunks per row
@@ -354,11 +356,12 @@ struct Decode8Tile {
   __device__ static __forceinline__ int off(int row, int c) { return row * D + 16 * (c ^ key(row)); }
 };
 
-// Four int8 as fp16 1152 + b: elements 0 and 2, then 1 and 3.
-__device__ __forceinline__ void i8x4_biased(uint32_t x, uint32_t& even, uint32_t& odd) {
+// Four int8 as fp16: elements 0 and 2, then 1 and 3.
+__device__ __forceinline__ void i8x4_f16(uint32_t x, uint32_t& even, uint32_t& odd) {
+  const f16x2_t bias = {static_cast<_Float16>(1152.0f), static_cast<_Float16>(1152.0f)};
   const uint32_t y = x ^ 0x80808080u;
-  even = perm_b32(0x64646464u, y, 0x04020400u);
-  odd = perm_b32(0x64646464u, y, 0x04030401u);
+  even = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2_t, perm_b32(0x64646464u, y, 0x04020400u)) - bias);
+  odd = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2_t, perm_b32(0x64646464u, y, 0x04030401u)) - bias);
 }
 
 // A16: cache rows start on 16 bytes (16-byte loads to LDS; else 4-byte ones).
@@ -374,8 +377,8 @@ __device__ __forceinline__ void decode8_segment(const DecodeArgs& a, lds_char_t*
   const int64_t unit = slot * a.hkv + kvh;
 
   // Q^T fragments: fragment 2m + u of this lane's head holds dims 64m + 16kg + 8u + {0, 2, 1, 3, 4, 6, 5, 7}
-  f16x8 qf[D / 32];
-  float sl, sc_off;  // score = S' * sl - sc_off
+  f16x8 qf[D / 32], ql[D / 32];  // the rounding, and 2^11 times the rest
+  float sl;                      // score = (S + 2^-11 S of the rest) * sl
   {
     const uint16_t* qh = a.q + (b * a.hq + kvh * a.g + (hcol < a.g ? hcol : 0)) * D;
     const float* ks = a.ksc + kvh * D;
@@ -395,21 +398,20 @@ __device__ __forceinline__ void decode8_segment(const DecodeArgs& a, lds_char_t*
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
     const int e2 = mx > 0.0f && mx < INFINITY ? max(-100, min(100, ilogbf(mx))) : 0;
-    float sum = 0.0f;
 #pragma unroll
     for (int f = 0; f < D / 32; ++f) {
-      _Float16 h[8];
+      _Float16 h[8], r[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        h[e] = static_cast<_Float16>(ldexpf(x[f][e], -e2));
-        sum += static_cast<float>(h[e]);
+        const float y = ldexpf(x[f][e], -e2);
+        h[e] = static_cast<_Float16>(y);
+        const float d = (y - static_cast<float>(h[e])) * 2048.0f;
+        r[e] = static_cast<_Float16>(fabsf(d) < INFINITY ? d : 0.0f);  // (nothing beside an infinity or a NaN)
       }
       qf[f] = f16x8{h[0], h[2], h[1], h[3], h[4], h[6], h[5], h[7]};
+      ql[f] = f16x8{r[0], r[2], r[1], r[3], r[4], r[6], r[5], r[7]};
     }
-    sum += __shfl_xor(sum, 16, 64);
-    sum += __shfl_xor(sum, 32, 64);
     sl = ldexpf(a.scale_log2, e2);
-    sc_off = 1152.0f * sum * sl;
   }
   f32x4 acc[D / 16];
 #pragma unroll
@@ -463,7 +465,6 @@ __device__ __forceinline__ void decode8_segment(const DecodeArgs& a, lds_char_t*
   };
   issue(0);
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(s_kv));
-  const f16x2_t bias2 = {static_cast<_Float16>(1152.0f), static_cast<_Float16>(1152.0f)};
   const f16x2_t ones = {static_cast<_Float16>(1.0f), static_cast<_Float16>(1.0f)};
   for (int s = 0; s < nsteps; ++s) {
     if (s + 1 < nsteps) {
@@ -494,17 +495,19 @@ __device__ __forceinline__ void decode8_segment(const DecodeArgs& a, lds_char_t*
     for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
       for (int m = 0; m < D / 64; ++m) asm volatile("" : "+v"(kr[tb][m]));
-    f32x4 sc[2];
+    f32x4 sc[2], sr[2];
 #pragma unroll
     for (int tb = 0; tb < 2; ++tb) {
       sc[tb] = f32x4{0, 0, 0, 0};
+      sr[tb] = f32x4{0, 0, 0, 0};
 #pragma unroll
       for (int f = 0; f < D / 32; ++f) {
         uint32_t o[4];
-        i8x4_biased(static_cast<uint32_t>(kr[tb][f >> 1][2 * (f & 1)]), o[0], o[1]);
-        i8x4_biased(static_cast<uint32_t>(kr[tb][f >> 1][2 * (f & 1) + 1]), o[2], o[3]);
-        sc[tb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, make_uint4(o[0], o[1], o[2], o[3])),
-                                                        qf[f], sc[tb], 0, 0, 0);
+        i8x4_f16(static_cast<uint32_t>(kr[tb][f >> 1][2 * (f & 1)]), o[0], o[1]);
+        i8x4_f16(static_cast<uint32_t>(kr[tb][f >> 1][2 * (f & 1) + 1]), o[2], o[3]);
+        const f16x8 kf = __builtin_bit_cast(f16x8, make_uint4(o[0], o[1], o[2], o[3]));
+        sc[tb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[f], sc[tb], 0, 0, 0);
+        sr[tb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, ql[f], sr[tb], 0, 0, 0);
       }
     }
     // lane: tokens 16tb + 4kg + r of head hcol
@@ -514,7 +517,7 @@ __device__ __forceinline__ void decode8_segment(const DecodeArgs& a, lds_char_t*
     for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float v = __builtin_fmaf(sc[tb][r], sl, -sc_off);
+        const float v = __builtin_fmaf(sr[tb][r], 0x1p-11f, sc[tb][r]) * sl;
         sc[tb][r] = 16 * tb + 4 * kg + r < left ? v : -INFINITY;
         mx = fmaxf(mx, sc[tb][r]);
       }
@@ -548,10 +551,8 @@ __device__ __forceinline__ void decode8_segment(const DecodeArgs& a, lds_char_t*
 #pragma unroll
     for (int t = 0; t < D / 16; ++t) {
       uint32_t o[4];
-      i8x4_biased(static_cast<uint32_t>(vr[t][0]), o[0], o[1]);
-      i8x4_biased(static_cast<uint32_t>(vr[t][1]), o[2], o[3]);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) o[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2_t, o[i]) - bias2);
+      i8x4_f16(static_cast<uint32_t>(vr[t][0]), o[0], o[1]);
+      i8x4_f16(static_cast<uint32_t>(vr[t][1]), o[2], o[3]);
       acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, make_uint4(o[0], o[1], o[2], o[3])), pf,
                                                       acc[t], 0, 0, 0);
     }
