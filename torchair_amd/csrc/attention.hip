@@ -1121,7 +1121,17 @@ __device__ __forceinline__ void prefill_item(const PrefillArgs& a, int64_t blk, 
       v_read(slot, std::integral_constant<int, 0>(), lo[0], hi[0]);
       v_read(slot, std::integral_constant<int, 1>(), lo[1], hi[1]);
       const float rs0 = softmax(s0, pf);
-      if (overflow(rs0)) continue;  // the next publish waits for the outstanding reads
+      // The value reads in flight keep their registers until they have landed: on the way out the compiler would take
+      // these as free and give them to, say, an address of the next tile's loads.
+      auto drain = [&] {
+#pragma unroll
+        for (int dt = 0; dt < D / 32; ++dt)
+          asm volatile("s_waitcnt lgkmcnt(0)" ::"v"(lo[0][dt]), "v"(hi[0][dt]), "v"(lo[1][dt]), "v"(hi[1][dt]) : "memory");
+      };
+      if (overflow(rs0)) {
+        drain();
+        continue;
+      }
       l_run += rs0;
       asm volatile("s_waitcnt lgkmcnt(%0)" ::"i"(kVReads) : "memory");
       pv_mfma(lo[0], hi[0], pf[0]);
@@ -1131,7 +1141,10 @@ __device__ __forceinline__ void prefill_item(const PrefillArgs& a, int64_t blk, 
         v_read(slot, std::integral_constant<int, 2>(), lo[0], hi[0]);
         v_read(slot, std::integral_constant<int, 3>(), lo[1], hi[1]);
         const float rs1 = softmax(s1, pf);
-        if (overflow(rs1)) continue;
+        if (overflow(rs1)) {
+          drain();
+          continue;
+        }
         l_run += rs1;
         asm volatile("s_waitcnt lgkmcnt(%0)" ::"i"(kVReads) : "memory");
         pv_mfma(lo[0], hi[0], pf[0]);
