@@ -1,7 +1,8 @@
 """tai_fia_tiled against tai_fia_general: every call the tiled kernels take is also the general kernel's, with
 the same arguments, so the two are run on the same inputs. Both keep scores, probabilities, sums and O in fp32
 precision and round the output once to 16 bits, so they differ by at most one rounding step of the output plus
-fp32 sums in another order: |a - b| <= 2^-7 |b| (bf16; 2^-10 fp16) + 2^-14 max|v|, and lse by 1e-4 of max(1, |lse|)."""
+fp32 sums in another order: |a - b| <= 2^-7 |b| (bf16; 2^-10 fp16) + 2^-14 max|v|, and lse by 1e-4 of max(1, |lse|).
+The last tests compare both kernels with 64-bit attention that shares none of their code."""
 import math
 
 import numpy as np
@@ -363,3 +364,61 @@ def test_mla_rows_workspace_follows_the_call(monkeypatch, lens, hq, sq, bs, most
     got, size = _guarded(monkeypatch, call)
     assert size <= most
     _assert_same(got, _both(monkeypatch, call)[1], 4.0)
+
+
+# ------------------------------------------------------------------------------------------------ against 64 bits
+def _attend64(q, k, v, scale):
+    """Bottom-right causal attention of q [lq, hq, dk] over k [lk, hkv, dk], v [lk, hkv, dv]: (out, lse)."""
+    lq, lk, rep = q.shape[0], k.shape[0], q.shape[1] // k.shape[1]
+    s = np.einsum("ihd,jhd->hij", q, np.repeat(k, rep, 1)) * scale
+    s = np.where(np.arange(lk)[None] <= np.arange(lq)[:, None] + lk - lq, s, -np.inf)
+    m = s.max(-1, keepdims=True)
+    p = np.exp(s - m)
+    l = p.sum(-1, keepdims=True)
+    return np.einsum("hij,jhd->ihd", p / l, np.repeat(v, rep, 1)), (m + np.log(l))[..., 0].T
+
+
+def _check64(out, lse, want, wlse, vmax, dt):
+    """One rounding of the output (8 significant bits round by up to 2^-8 of the value, 11 by 2^-11), P as a 16-bit
+    pair (2^-17 of a term) and fp32 scores and sums, 2^-15 of the largest value in all."""
+    u = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -11
+    far = np.abs(out.double().cpu().numpy() - want) - 1.01 * u * np.abs(want)
+    assert far.max() <= 2.0 ** -15 * vmax
+    assert np.abs((lse.double().cpu().numpy() - wlse) / np.maximum(1, np.abs(wlse))).max() <= 1e-5
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hkv,d,bs", [(8, 2, 128, 64), (7, 1, 128, 96), (4, 4, 64, 32)])
+def test_packed_against_64_bits(monkeypatch, hq, hkv, d, bs, dt):
+    g = torch.Generator().manual_seed(400 + hq)
+    lq, lk = [1, 70, 5, 1, 33], [700, 70, 260, 1, 900]
+    bt, n = _table(lk, bs, g)
+    k, v = _kv(n, bs, hkv, d, dt, g)
+    q = (torch.randn(sum(lq), hq, d, generator=g) * 2).to(dt).to(DEV)
+    both = _both(monkeypatch, lambda: FIA(
+        q, k, v, actual_seq_lengths=torch.tensor(np.cumsum(lq), device=DEV),
+        actual_seq_lengths_kv=torch.tensor(lk, device=DEV), block_table=bt.to(DEV), num_heads=hq,
+        num_key_value_heads=hkv, input_layout="TND", block_size=bs, scale=d ** -0.5, sparse_mode=3, softmax_lse_flag=True))
+    q, k, v = [x.double().cpu().numpy() for x in (q, k, v)]
+    at = 0
+    for i, (a, b) in enumerate(zip(lq, lk)):
+        pages = bt[i, :-(-b // bs)].numpy()
+        kk, vv = [x[pages].reshape(-1, hkv, d)[:b] for x in (k, v)]
+        want, wlse = _attend64(q[at:at + a], kk, vv, d ** -0.5)
+        for out, lse in both:
+            _check64(out[at:at + a], lse[at:at + a].reshape(a, hq), want, wlse, np.abs(vv).max(), dt)
+        at += a
+
+
+@pytest.mark.parametrize("hq,sq", [(16, 1), (40, 3), (130, 1)])
+def test_mla_rows_against_64_bits(monkeypatch, hq, sq):
+    lens, bs = [sq, 33, 260, 700], 32
+    t = _mla(lens, hq, sq, bs, 410 + hq)
+    both = _both(monkeypatch, _mla_call(t, lens, hq, bs, sparse_mode=3))
+    qn, qr, c, kr, bt = [x.double().cpu().numpy() for x in t]
+    for i, n in enumerate(lens):
+        pages = bt[i, :-(-n // bs)].astype(int)
+        cc, rr = c[pages].reshape(-1, 1, 512)[:n], kr[pages].reshape(-1, 1, 64)[:n]
+        want, wlse = _attend64(np.concatenate([qn[i], qr[i]], -1), np.concatenate([cc, rr], -1), cc, 192 ** -0.5)
+        for out, lse in both:
+            _check64(out[i], lse[i].reshape(hq, sq).T, want, wlse, np.abs(cc).max(), torch.bfloat16)

@@ -408,6 +408,53 @@ def test_compiled_int8_cache_and_sink_decode_replay_with_new_lengths():
         assert tai_graph.stats["eager_fallbacks"] == falls
 
 
+def test_compiled_packed_and_bf16_mla_replay_with_new_lengths():
+    """The tiled attention kernels, which plan on the device: packed queries over a paged cache and MLA over a bf16
+    latent (one and two query tokens), captured once; each replay, with new lengths, ends and block tables, equals
+    the eager call. Empty sequences, rows past the last end and calls of one long sequence come in turn."""
+    g = torch.Generator().manual_seed(55)
+    b, t, hq, hkv, d, bs, width = 6, 40, 8, 2, 64, 32, 12
+    nblk = b * width
+    kc, vc = [torch.randn(nblk, bs, hkv * d, generator=g).to(torch.bfloat16).to(DEV) for _ in range(2)]
+    lat = torch.randn(nblk, bs, 1, 512, generator=g).to(torch.bfloat16).to(DEV)
+    kr = torch.randn(nblk, bs, 1, 64, generator=g).to(torch.bfloat16).to(DEV)
+
+    def packed(q, ends, lens, bt):
+        return torch.ops.air.npu_fused_infer_attention_score(
+            q, kc, vc, actual_seq_lengths=ends, actual_seq_lengths_kv=lens, block_table=bt, num_heads=hq,
+            num_key_value_heads=hkv, input_layout="TND", block_size=bs, scale=d ** -0.5, sparse_mode=3)[0]
+
+    def mla(q, qr, lens, bt):
+        return torch.ops.air.npu_fused_infer_attention_score(
+            q, lat, lat, query_rope=qr, key_rope=kr, actual_seq_lengths_kv=lens, block_table=bt, num_heads=hq,
+            num_key_value_heads=1, input_layout="BSND", block_size=bs, scale=192 ** -0.5, sparse_mode=3)[0]
+
+    def half(*shape):
+        return torch.randn(*shape, generator=g).to(torch.bfloat16).to(DEV)
+
+    for name, step, sq in (("packed", packed, 0), ("mla", mla, 1), ("mla", mla, 2)):
+        fn = torch.compile(step, backend=_backend(), fullgraph=True)
+        torch._dynamo.reset()
+        caps, falls = tai_graph.stats["captures"], tai_graph.stats["eager_fallbacks"]
+        for i in range(5):
+            lens = torch.randint(max(1, sq), width * bs + 1, (b,), generator=g)
+            ends = torch.randint(0, t + 1, (b,), generator=g).sort().values
+            if i == 2:
+                lens[1], lens[4] = 0, 1
+            if i == 3:  # one sequence holds everything
+                lens[:], ends[:] = 0, 0
+                lens[5], ends[5] = width * bs, t
+            bt = _paged(g, lens.tolist(), nblk, width, bs, hkv, d).to(DEV)
+            print("case", name, sq, "replay", i, flush=True)
+            args = [half(t, hq, d), ends.to(DEV)] if name == "packed" else [half(b, sq, hq, 512), half(b, sq, hq, 64)]
+            args += [lens.to(DEV), bt]
+            got = fn(*args).clone()
+            assert torch.equal(got, step(*args)), f"{name} {sq}: replay {i} differs from eager"
+            _churn()
+        assert tai_graph.stats["captures"] == caps + 1
+        assert tai_graph.stats["eager_fallbacks"] == falls
+
+
 def _cyclic_runner(x):
     """A captured runner whose function refers back to what holds it."""
     held = {}
