@@ -238,7 +238,8 @@ def fia_cuda(query, key, value, **kw):
     seq_q = _lens_tensor(kw.get("actual_seq_lengths"), query.device)
 
     mask_origin, pre, nxt, explicit = _mask_params(kw)
-    # int8 key / value caches (GQA / MHA) and int8 attention_out take the general kernel
+    # int8 attention_out and int8 key / value caches (GQA / MHA) take the general kernel, but for one token over a paged
+    # cache with per-channel scales (below)
     quant_out = kw.get("quant_scale2") is not None
     kv8 = key.dtype == torch.int8 and kw.get("query_rope") is None
     qq = query.dtype == torch.int8
@@ -265,7 +266,7 @@ def fia_cuda(query, key, value, **kw):
     sink = kw.get("learnable_sink")  # (the v2 op's input)
     _check(sink is None or not qq, "npu_fused_infer_attention_score: learnable_sink is not served with an int8 query")
     # a sink with nothing else also runs on the one-token decode kernel (its merge takes the sink in);
-    # every other case with a prefix or a sink takes the general kernel
+    # every other case with a prefix or a sink goes through _general_call
     sink_only = pse is None and not prefix and sink is not None
     pse = pse if pse is not None else (True if prefix or sink is not None else None)
     _check(kw.get("quant_offset2") is None or quant_out, "npu_fused_infer_attention_score: quant_offset2 needs "
@@ -301,7 +302,7 @@ def fia_cuda(query, key, value, **kw):
             if (key.dtype == torch.int8 and s == 1 and whole_prefix and not explicit and key.size(1) % 32 == 0
                     and not packed and sink is None):
                 return _mla(query, key, value, kw, out, lse, want_lse, num_heads, n_kv, bt, seq_kv, scale, stream)
-            # several query tokens (MTP / speculative decode), bands and masks: the general kernel
+            # a bf16 / fp16 latent; several query tokens (MTP / speculative decode), bands and masks
             return _general_mla(query, key, value, kw, out, lse, want_lse, ql, num_heads, n_kv, bt, seq_q, seq_kv,
                                 scale, mask_origin, pre, nxt, explicit, stream, ol=ol)
         dt = _half_code(query, key, value, kv8)
@@ -631,8 +632,9 @@ def _packed_lens(a, ql, query, bt, seq_q, seq_kv):
 
 def _general_call(query, key, value, out, lse, want_lse, ql, num_heads, n_kv, d, dt, ks, vs, bt, bs, seq_q, seq_kv,
                   mask_origin, pre, nxt, explicit, kw, scale, stream, kv8=False, quant_out=False, ol=None):
-    """The general kernel for GQA/MHA: explicit masks, head dims the tiled kernels do not take, int8
-    key/value caches, int8 attention_out and packed (TND / NTD) queries."""
+    """GQA/MHA calls described by tai_fia_general_args. The tiled kernels take those that tai_fia_tiled_workspace_size
+    names (packed TND / NTD queries and batched ones with a sink, 64 or 128 dims); explicit masks, pse_shift, a shared
+    prefix, other head dims, int8 keys/values and int8 attention_out are left to the general kernel."""
     ol = ol or ql
     packed = ql in _PACKED
     if packed:
@@ -705,9 +707,11 @@ def _launch_general(a, device, stream):
 
 def _general_mla(query, key, value, kw, out, lse, want_lse, ql, num_heads, n_kv, bt, seq_q, seq_kv, scale,
                  mask_origin, pre, nxt, explicit, stream, ol=None):
-    """MLA on the general kernel: key = [latent | key_rope], value = latent, one kv head. The latent is
-    bf16 / fp16, or int8 with one fp32 scale per cache slot (key_antiquant_scale [blocks, bs],
-    key_antiquant_mode 1, as for the one-token kernel), then dequantised as latent * scale."""
+    """MLA calls described by tai_fia_general_args: key = [latent | key_rope], value = latent, one kv head. The latent
+    is bf16 / fp16, or int8 with one fp32 scale per cache slot (key_antiquant_scale [blocks, bs],
+    key_antiquant_mode 1, as for the one-token kernel), then dequantised as latent * scale. The tiled kernels take a
+    bf16 latent without a lower bound or an explicit mask, in pages of whole 32-token steps; the rest is left to the
+    general kernel."""
     q_rope, k_rope = kw["query_rope"], kw.get("key_rope")
     _check(k_rope is not None, "npu_fused_infer_attention_score: MLA needs key_rope")
     _check(n_kv == 1, "npu_fused_infer_attention_score: MLA latent cache has one kv head")
@@ -832,7 +836,7 @@ def _mla(query, key, value, kw, out, lse, want_lse, num_heads, n_kv, bt, seq_kv,
 # under renamed arguments, lowered to the same FusedInferAttentionScore node (:166-181), so it maps onto
 # the v1 implementation argument for argument. Arguments of v2 with no v1 counterpart that this build
 # does not serve (query quantisation, the softmax quant scale, dtype reinterpretations) are refused;
-# learnable_sink is passed on to the v1 implementation, which serves it on the general kernel.
+# learnable_sink is passed on to the v1 implementation.
 _V2_UNSUPPORTED = ("dequant_scale_query", "quant_scale_p", "query_dtype", "key_dtype", "value_dtype",
                    "query_rope_dtype", "key_rope_dtype", "key_shared_prefix_dtype", "value_shared_prefix_dtype",
                    "dequant_scale_query_dtype", "dequant_scale_key_dtype", "dequant_scale_value_dtype",

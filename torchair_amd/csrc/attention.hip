@@ -580,10 +580,10 @@ void paged_decode8_kernel(DecodeArgs a) {
 }
 
 // Merge the partials of (b, q head) pairs, WPH waves per head, each lane owning D / 64 consecutive d. The
-// partials are those of the ranges that cover the sequence's steps; wave i of a head takes every WPH-th. A partial's statistics are wave-uniform loads, and the loads of four partials go
-// out together. WPH follows the partials a sequence has on average (ranges / sequences): one wave walks up to 8
-// of them; with 43 each (3 sequences of 3000-20000 tokens) it took 26 us where the decode kernel took 24, sixteen
-// take 5.
+// partials are those of the ranges that cover the sequence's steps; wave i of a head takes every WPH-th. A partial's
+// statistics are wave-uniform loads, and the loads of four partials go out together. WPH follows the partials a
+// sequence has on average (ranges / sequences): one wave walks up to 8 of them; with 43 each (3 sequences of
+// 3000-20000 tokens) it took 26 us where the decode kernel took 24, sixteen take 7.
 template <int D, bool F16, int WPH>
 __global__ __launch_bounds__(64 * (WPH < 4 ? 4 : WPH)) void decode_combine_kernel(DecodeArgs a, uint16_t* out, float* lse) {
   constexpr int E = D / 64;  // outputs per lane

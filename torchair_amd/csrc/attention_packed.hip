@@ -9,12 +9,14 @@
 // LDS ring, two tiles ahead (the tile layout and fragment reads of the prefill kernel).
 //
 // Sequence lengths are on the device, so the launch is one workgroup per CU over equal ranges of the items' cost
-// (planned by packed_plan_kernel): long prompts, short chunks and single tokens fill the chip alike. An item cut
-// by a range's end leaves fp32 partials, which packed_merge_kernel joins.
+// (planned by the kernel itself, or by packed_plan_kernel where sequences are many or long): long prompts, short
+// chunks and single tokens fill the chip alike. An item cut by a range's end leaves fp32 partials, which
+// packed_merge_kernel joins.
 //
 // Measured (6 chunks of 128-512 tokens and 24 single tokens over contexts up to 4096, 32 / 8 heads of 128):
-// 26.1 ms on the general kernel (each row and head read its keys and values alone), 0.208 ms here: plan 7 us,
-// this kernel 185, merge 16. Its MFMAs (48 per wave and tile, a third of them for lo) take about 100 us.
+// 26.1 ms on the general kernel (each row and head read its keys and values alone), 0.202 ms here: plan 6 us, merge
+// 14, the rest this kernel. Its MFMAs (48 per wave and tile, a third of them for lo) take about 100 us; they are 27%
+// busy, the vector units 31%, HBM at 2.2 TB/s: score, softmax and P.V of a tile follow one another.
 #include "attention_common.h"
 
 namespace tai {
@@ -109,8 +111,9 @@ __device__ __forceinline__ int64_t seq_cost(const PackedArgs& p, int64_t b) {
   return c;
 }
 
-// A lane per sequence, so that many short ones are planned at once (a wave each took 23 us for 256 single tokens, beside 39 of the main kernel);
-// a sequence of many blocks is summed by its whole wave. Neighbouring sequences go to different waves.
+// A lane per sequence, so that many short ones are planned at once (a wave each took 23 us for 256 single tokens,
+// beside 39 of the main kernel); a sequence of many blocks is summed by its whole wave. Neighbouring sequences go to
+// different waves.
 __global__ __launch_bounds__(1024) void packed_plan_kernel(PackedArgs p) {
   __shared__ int64_t red[16];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -505,8 +508,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int64_t* pref = p.pref;
   if (p.plan_here) {
     // a thread per sequence; the plan kernel and its launch cost small calls more (4 tokens over 64: 15.8 us with it,
-    // 13.1 without; 256 single tokens over 64, 16 / 8 heads of 64: 64 and 41 us). Up to 64 sequences one wave does it, which saves the others'
-    // part of the scan, 0.4 us.
+    // 13.1 without; 256 single tokens over 64, 16 / 8 heads of 64: 64 and 41 us). Up to 64 sequences one wave does
+    // it, which saves the others' part of the scan, 0.4 us.
     if (p.a.b > 64 || threadIdx.x < 64) {
       const int64_t c = threadIdx.x < p.a.b ? seq_cost(p, threadIdx.x) * p.a.hkv : 0;
       const int64_t incl = p.a.b > 64 ? block_incl_scan<false>(c, red) : wave_incl_scan64(c, lane);

@@ -1,9 +1,10 @@
 // Tiled MFMA kernels for attention whose probabilities stay in fp32 precision: the MLA latent cache in
-// bf16 (here), and GQA/MHA query blocks (attention_packed.hip). They take over from the general kernel (attention_general.hip) the calls
-// tai_fia_tiled_workspace_size() names; the arguments and the meaning of every field are that kernel's.
+// bf16 (here), and GQA/MHA query blocks (attention_packed.hip). They take over from the general kernel
+// (attention_general.hip) the calls tai_fia_tiled_workspace_size() names; the arguments and the meaning of
+// every field are that kernel's.
 //
 // P enters the P.V MFMA as a bf16 pair, hi = bf16(p) and lo = bf16(p - hi): hi + lo carries 16 bits of p's
-// mantissa, so the products' error is 2^-17 of a term, below the output's own rounding (2^-9). Scores, row
+// mantissa, so the products' error is 2^-17 of a term, below the output's own rounding (2^-8). Scores, row
 // sums, O and the partial results are fp32, as in the general kernel.
 #include "attention_common.h"
 
@@ -59,7 +60,7 @@ __device__ __forceinline__ RowInfo row_info(const tai_fia_general_args& a, int64
 // range's end leaves fp32 partials that mla_rows_merge_kernel joins, any other row is written here.
 //
 // Measured (32 sequences of 512-4096 tokens, 128 heads): 5.2 ms on the general kernel (a wave per row and head,
-// nothing shared), 66 us here, of which the merge 14. A step takes 3.4 us against 1.4 us of MFMAs (100 per
+// nothing shared), 67 us here, of which the merge 13. A step takes 3.4 us against 1.4 us of MFMAs (100 per
 // SIMD: 36 score, 64 P.V) because its score, softmax and P.V phases follow one another between the barriers;
 // a segment costs about 25 us on top (query fragments, ring fill, 256 KB of partial per workgroup).
 constexpr int kRStep = 32;
@@ -584,7 +585,8 @@ bool mla_rows_takes(const tai_fia_general_args& a) {
          a.v_strides[1] == a.k1_strides[1] && a.pre_tokens >= (int64_t(1) << 31) - 1 && a.q1 && a.q2 && a.k1 && a.k2 &&
          a.out && aligned(a.q1, 16) && aligned(a.q2, 16) && aligned(a.k1, 16) && aligned(a.k2, 16) && aligned(a.out, 8) &&
          rows_aligned(a.q1_strides, 8) && rows_aligned(a.q2_strides, 8) && rows_aligned(a.k1_strides, 8) &&
-         rows_aligned(a.k2_strides, 8) && small_row(a.k1_strides[1]) && small_row(a.k2_strides[1]) && rows_aligned(a.out_strides, 4) && query_rows(a) <= (int64_t(1) << 18) &&
+         rows_aligned(a.k2_strides, 8) && small_row(a.k1_strides[1]) && small_row(a.k2_strides[1]) &&
+         rows_aligned(a.out_strides, 4) && query_rows(a) <= (int64_t(1) << 18) &&
          query_rows(a) * a.hq < (int64_t(1) << 31);
 }
 
