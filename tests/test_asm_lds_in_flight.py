@@ -84,7 +84,7 @@ def touched_in_flight(lines, only_past=None):
     return sorted(found)
 
 
-def test_the_checker_itself():
+def test_the_scan_sees_reads_left_in_flight():
     read = [";;#ASMSTART", "ds_read_b128 v[4:7], v1", ";;#ASMEND"]
     wait = [";;#ASMSTART", "s_waitcnt lgkmcnt(0)", ";;#ASMEND"]
     use = ["v_add_f32_e32 v0, v4, v5", "s_endpgm"]
